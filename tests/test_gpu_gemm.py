@@ -251,6 +251,24 @@ def test_gemm_f16_nn(dev, M, N, K, pad, out):
         assert bool(torch.all((c[:M].double() - ref).abs() <= bound))
 
 
+@pytest.mark.parametrize("N,ldb", [(77, 80), (1001, 1008), (1002, 1008), (1004, 1008), (193, 200)])
+@pytest.mark.parametrize("M,K", [(130, 72), (300, 768)])
+def test_wmma_matmul_column_slice(dev, M, K, N, ldb):
+    """B[K,N] with N off 8 in rows of a wider pitch (a column slice): its last
+    row ends inside a 16-byte vector, and inside a 4-byte word for odd N. That
+    row carries the result (the others are 2^-10 of it), so a lost term shows."""
+    from zenith_amd import zenith_cuda as zc
+
+    g = torch.Generator(device=dev).manual_seed(N)
+    a = torch.randn(M, K, generator=g, device=dev).half()
+    wide = torch.randn(K, ldb, generator=g, device=dev).half()
+    wide[:-1] *= 2.0**-10
+    c = zc.wmma_matmul(a, wide[:, :N])
+    a64, b64 = a.double(), wide[:, :N].double().contiguous()
+    bound = K * 2.0**-24 * (a64.abs() @ b64.abs())
+    assert bool(torch.all((c.double() - a64 @ b64).abs() <= bound))
+
+
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("M,N,K,pad", [
     (64, 1100, 1600, 0),   # 64x64 tile, K split, K a multiple of 32

@@ -419,11 +419,15 @@ void gemm_mfma_kernel(GemmParams p) {
           : (void *)((const char *)p.A + (int64_t)m0 * lda_b),
       (short)0, APK ? a_blocks * (kbytes / 32) * 1024 : (int)((a_rows - 1) * lda_b + kbytes),
       0x00020000);
-  // BNK: B is [K,N], its descriptor ends with the last row (rows past K read
-  // as zero; columns past N read what follows and are not stored)
+  // BNK: B is [K,N], its descriptor ends with the 16-byte vector that holds the
+  // last row's last column (inside the row's pitch, a multiple of 8): a 4-byte
+  // word that straddles the end reads as zero, which for odd N would drop
+  // that column's last product. Rows past K read as zero; columns past N read
+  // what follows and are not stored.
   const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(
       (void *)((const char *)p.B + (BNK ? (int64_t)n0 * 2 : (int64_t)n0 * ldb_b)), (short)0,
-      BNK ? (int)((p.K - 1) * ldb_b + (int64_t)(p.N - n0) * 2) : (int)((b_rows - 1) * ldb_b + kbytes),
+      BNK ? (int)((p.K - 1) * ldb_b + (int64_t)(((p.N + 7) & ~7) - n0) * 2)
+          : (int)((b_rows - 1) * ldb_b + kbytes),
       0x00020000);
 
   // DMA source offsets. Instruction g of this wave fills tile rows
