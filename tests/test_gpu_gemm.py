@@ -269,6 +269,20 @@ def test_wmma_matmul_column_slice(dev, M, K, N, ldb):
     assert bool(torch.all((c.double() - a64 @ b64).abs() <= bound))
 
 
+def test_matmul_fp32_many_rows(dev):
+    """More rows than a 16-bit count of 64-row tiles holds."""
+    from zenith_amd import zenith_cuda as zc
+
+    M, K, N = 65535 * 64 + 69, 8, 32
+    g = torch.Generator(device=dev).manual_seed(3)
+    a, b = torch.randn(M, K, generator=g, device=dev), torch.randn(K, N, generator=g, device=dev)
+    c = zc.matmul(a, b)
+    for rows in (slice(0, 64), slice(65535 * 64 - 64, M)):
+        a64 = a[rows].double()
+        bound = K * 2.0**-24 * (a64.abs() @ b.double().abs())
+        assert bool(torch.all((c[rows].double() - a64 @ b.double()).abs() <= bound))
+
+
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("M,N,K,pad", [
     (64, 1100, 1600, 0),   # 64x64 tile, K split, K a multiple of 32

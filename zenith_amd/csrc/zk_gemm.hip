@@ -836,8 +836,6 @@ static int gemm_f32_impl(const float *A, const float *B, float *C, int64_t M, in
   const bool matrix = trans_b && K > 0 && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
                       aligned16(A) && aligned16(B) &&
                       255 * (lda + ldb) * 4 + 2 * K * 4 < 0x7ffffff0LL;
-  if (!matrix && (M + 63) / 64 > 65535)
-    return fail(ZK_ERR_UNSUPPORTED, "zk_gemm_f32: M too large");
   // the bf16-split kernel's offsets: 128 rows of A or W, 32 rows of B[K,N]
   const bool span = 127 * lda * 4 + K * 4 < 0x7ffffff0LL &&
                     (trans_b ? 127 * ldb * 4 + K * 4 : 31 * ldb * 4 + N * 4) < 0x7ffffff0LL;
@@ -859,6 +857,8 @@ static int gemm_f32_impl(const float *A, const float *B, float *C, int64_t M, in
       ok = launch_mfma<F32Op, float, false>(p, epi, s);
     return launched(ok, who, epi);
   }
+  if ((M + 63) / 64 > 65535)  // the SIMT kernel's grid; the others' have one dimension
+    return fail(ZK_ERR_UNSUPPORTED, "%s: M too large", who);
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
   if (trans_b)
     gemm_f32_kernel<true><<<grid, 256, 0, s>>>(A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc);
