@@ -274,3 +274,17 @@ def test_attention_fp16_gpu_matches_converted(dev, B, H, S, D):
     assert torch.equal(torch.isfinite(got), torch.isfinite(ref))
     ok = torch.isfinite(ref)
     torch.testing.assert_close(got[ok], ref[ok], rtol=2.0**-10, atol=2.0**-24)
+
+
+def test_attention_fp16_gpu_odd_batch_pitch(dev):
+    """A batch of one whose (unused) batch stride is no multiple of 4: contiguous
+    for torch, and computed as any other."""
+    from zenith_amd import core_cuda as cuda
+
+    H, S, D = 3, 5, 64
+    buf = torch.from_numpy(synthetic.normal((2048,), tag=70)).to(dev)
+    t = buf.as_strided((1, H, S, D), (H * S * D + 1, S * D, D, 1))
+    g = cuda.GpuTensor(t)
+    ref = cuda.GpuTensor(t.clone(memory_format=torch.contiguous_format).reshape(1, H, S, D))
+    got = cuda.attention_fp16_gpu(g, g, g).tensor
+    assert torch.equal(got, cuda.attention_fp16_gpu(ref, ref, ref).tensor)

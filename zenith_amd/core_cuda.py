@@ -205,7 +205,9 @@ def _attn_fp16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> GpuTensor:
     """fp16 attention on fp32 tensors: one launch for up to 128 queries of
     dim 64, else converted, computed and converted back."""
     B, H, S, D = q.shape
-    if D == 64 and S <= 128 and all(t.data_ptr() % 16 == 0 for t in (q, k, v)):
+    # contiguous by GpuTensor; a dimension of one may carry any stride all the same
+    if D == 64 and S <= 128 and all(t.data_ptr() % 16 == 0 and
+                                    all(d % 4 == 0 for d in t.stride()[:3]) for t in (q, k, v)):
         o = _new(q)
         strides = L.strides_arg([*q.stride()[:3], *k.stride()[:3], *v.stride()[:3],
                                  *o.stride()[:3]])
