@@ -348,6 +348,65 @@ def test_gemm_f32_bf16_split_special_values(dev, trans_b):
     assert np.all(np.abs(got[ok] - ref[ok]) <= K * 2.0**-24 * mag[ok])
 
 
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("exp_a,exp_b", [(-116, 40), (-124, 60), (-130, 100), (-62, -40), (30, -146)])
+def test_gemm_f32_bf16_split_small_values(dev, trans_b, exp_a, exp_b):
+    """Operands down to fp32's subnormals through the bf16-split GEMM: every
+    fp32 value is split exactly, so the bar is that of ordinary values, the
+    result's own last subnormal place beside it."""
+    from zenith_amd import _lib as L
+
+    M, N, K = 1100, 1100, 136
+    rng = np.random.default_rng([1000 + exp_a, 1000 + exp_b])
+    a = np.ldexp(rng.standard_normal((M, K)), exp_a).astype(np.float32)
+    b = np.ldexp(rng.standard_normal((K, N)), exp_b).astype(np.float32)
+    ta, tb = _t(a, dev, torch.float32), _t(b.T if trans_b else b, dev, torch.float32)
+    c = torch.empty((M, N), device=dev)
+    L.call("zk_gemm_f32", ta.data_ptr(), tb.data_ptr(), c.data_ptr(), M, N, K, K,
+           K if trans_b else N, N, int(trans_b), torch.cuda.current_stream().cuda_stream)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    bound = K * 2.0**-24 * (np.abs(a64) @ np.abs(b64)) + 2.0**-149
+    assert np.all(np.abs(c.cpu().numpy() - a64 @ b64) <= bound)
+
+
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("N", [1100, 1030])  # rows of whole 16-byte vectors, and not
+@pytest.mark.parametrize("K", [40, 3201])  # one slice and a tail; K split
+def test_gemm_f32_bf16_split_large_values(dev, trans_b, N, K):
+    """Sums and products up to FLT_MAX: finite wherever fp32's are, and infinite
+    where the result is past its range. Rows 0 to 127 hold products within 2^-9
+    of FLT_MAX whose factors' leading bf16 parts multiply past it."""
+    from zenith_amd import _lib as L
+
+    M, fmax = 1100, float(np.finfo(np.float32).max)
+    rng = np.random.default_rng(K)
+    a = np.ldexp(rng.uniform(1, 2, (M, K)), rng.integers(40, 58, (M, 1))).astype(np.float32)
+    b = np.ldexp(rng.uniform(-2, 2, (K, N)), rng.integers(40, 58, (1, N))).astype(np.float32)
+    a[:128] = 0
+    a[:128, 7] = np.float32(1.99609387 * 2.0**63)  # rounds up to 1.9975586 * 2^63 or more
+    b[7, :] = (fmax * (1 - rng.uniform(2.0**-11, 2.0**-9, N)) / a[0, 7]).astype(np.float32)
+    a[128, 3], a[129, 5] = 3.4e38, -3.4e38
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    ref = a64 @ b64
+    bound = K * 2.0**-24 * (np.abs(a64) @ np.abs(b64))
+    sure = np.abs(ref) + bound < fmax  # finite in any order of the sums, unless an
+    sure &= np.abs(a64) @ np.abs(b64) < fmax  # intermediate sum overflows
+    assert sure[:128].all()
+    n = int(L.load().zk_gemm_workspace_size(M, N, K, L.ZK_F32))
+    ws = torch.empty(max(n, 16), dtype=torch.uint8, device=dev)
+    ta, tb = _t(a, dev, torch.float32), _t(b.T if trans_b else b, dev, torch.float32)
+    for nbytes in {0, n}:
+        c = torch.empty((M, N), device=dev)
+        L.call("zk_gemm_f32_ws", ta.data_ptr(), tb.data_ptr(), c.data_ptr(), M, N, K, K,
+               K if trans_b else N, N, int(trans_b), ws.data_ptr(), nbytes,
+               torch.cuda.current_stream().cuda_stream)
+        got = c.cpu().numpy().astype(np.float64)
+        assert np.isfinite(got[sure]).all()
+        assert np.all(np.abs(got[sure] - ref[sure]) <= bound[sure])
+        past = np.abs(ref) - bound > fmax * (1 + 2.0**-24)
+        assert not np.isfinite(got[past]).any()
+
+
 def test_linear_fp32(dev):
     from zenith_amd import zenith_cuda as zc
 
