@@ -275,6 +275,42 @@ def test_flash_attention_f32(dev, B, H, S, D, masked):
     np.testing.assert_allclose(o, ops.attention(q, k, v, lens), rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("B,H", [(16, 32), (10, 10), (2, 1)])  # keys split 1, 2 and 4 ways
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("masked", [False, True])
+def test_flash_attention_f32_small_probabilities(dev, B, H, D, masked):
+    """Keys whose probability is an fp32 subnormal still count where their V is
+    large: e^-88 2^40 of a key beside a key of V = 0, in the same stage and in
+    a later one, before the key that sets the maximum, and last of the valid
+    ones. Masked (batch 0), or past the valid length (the last batch), it does not."""
+    from zenith_amd import zenith_cuda as zc
+
+    S = 128
+    q = torch.zeros(B, H, S, D, device=dev)
+    k, v = torch.zeros_like(q), torch.zeros_like(q)
+    q[..., 0] = 8.0
+    for small in (1, 20, 70, 99, 0):
+        top = 2 if small == 0 else 0
+        k.zero_(), v.zero_()
+        k[..., 0] = -400.0  # every other key: probability 0
+        k[:, :, top, 0], k[:, :, small, 0] = 0.0, -88.0
+        v[:, :, small] = 2.0**40
+        ref = torch.full_like(q, math.exp(-88.0) * 2.0**40)
+        kw = {}
+        if masked:
+            mask = torch.ones(B, 1, S, S, dtype=torch.bool, device=dev)
+            mask[0, :, :, small] = False
+            kw["attn_mask"] = mask
+            ref[0] = 0.0
+        lens = torch.full((B,), 100, dtype=torch.int32, device=dev)
+        if small > 2:
+            lens[-1] = small
+            ref[-1] = 0.0
+        o = zc.flash_attention(q, k, v, scale=0.125, key_padding_lengths=lens, **kw)
+        # a subnormal near 2^-127 is known to 2^-149 / 2, the score to 88 2^-23
+        torch.testing.assert_close(o, ref, rtol=2e-5, atol=0)
+
+
 @pytest.mark.parametrize("B,H", [(16, 32), (10, 10), (2, 3)])  # keys split 1, 2 and 4 ways
 @pytest.mark.parametrize("D,pitch", [(64, 64), (64, 65), (96, 96), (33, 33)])
 def test_flash_attention_f32_key_split(dev, B, H, D, pitch):

@@ -83,6 +83,9 @@ __device__ __forceinline__ int valid_len(const AttnParams &p, int b) {
 __device__ __forceinline__ float smax(float a, float b) {
   return __builtin_amdgcn_fmed3f(a, b, __builtin_inff());
 }
+__device__ __forceinline__ float smin(float a, float b) {
+  return __builtin_amdgcn_fmed3f(a, b, -__builtin_inff());
+}
 
 // ds_read_b64_tr_b16: 8 bytes per lane, transposed across each group of 16
 // lanes (see its use below for the lane mapping).
