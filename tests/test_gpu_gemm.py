@@ -283,6 +283,21 @@ def test_matmul_fp32_many_rows(dev):
         assert bool(torch.all((c[rows].double() - a64 @ b.double()).abs() <= bound))
 
 
+@pytest.mark.parametrize("M,K", [(3, 9), (65, 41)])  # SIMT and bf16-split kernels
+def test_matmul_fp32_wide_b(dev, M, K):
+    """Rows of B so wide that 32 of them pass 2^31 bytes (8 do not)."""
+    from zenith_amd import zenith_cuda as zc
+
+    N = 17_400_001
+    g = torch.Generator(device=dev).manual_seed(4)
+    a, b = torch.randn(M, K, generator=g, device=dev), torch.randn(K, N, generator=g, device=dev)
+    c = zc.matmul(a, b)
+    for cols in (slice(0, 200), slice(N // 2, N // 2 + 200), slice(N - 200, N)):
+        b64 = b[:, cols].double().contiguous()
+        bound = K * 2.0**-24 * (a.double().abs() @ b64.abs())
+        assert bool(torch.all((c[:, cols].double() - a.double() @ b64).abs() <= bound))
+
+
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("M,N,K,pad", [
     (64, 1100, 1600, 0),   # 64x64 tile, K split, K a multiple of 32

@@ -836,9 +836,13 @@ static int gemm_f32_impl(const float *A, const float *B, float *C, int64_t M, in
   const bool matrix = trans_b && K > 0 && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
                       aligned16(A) && aligned16(B) &&
                       255 * (lda + ldb) * 4 + 2 * K * 4 < 0x7ffffff0LL;
-  // the bf16-split kernel's offsets: 128 rows of A or W, 32 rows of B[K,N]
+  // the bf16-split kernel's offsets: 128 rows of A or W, 8 rows of B[K,N]. Where
+  // 32 rows of B pass 31 bits (N above 17 million) few rows stay on the SIMT
+  // kernel: M x K x 17.4e6, SIMT / split: 2 x 8 0.6 / 2.0 ms, 64 x 64 4.1 / 3.5,
+  // 256 x 64 16.3 / 8.4.
   const bool span = 127 * lda * 4 + K * 4 < 0x7ffffff0LL &&
-                    (trans_b ? 127 * ldb * 4 + K * 4 : 31 * ldb * 4 + N * 4) < 0x7ffffff0LL;
+                    (trans_b ? 127 * ldb * 4 + K * 4
+                             : (M < 64 ? 31 : 7) * ldb * 4 + N * 4) < 0x7ffffff0LL;
   const F32Plan fp =
       span ? plan_f32s(M, N, K, matrix ? F32Other::kMatrix : F32Other::kFma) : F32Plan{0, 1, 0};
   if (fp.tile) {
