@@ -288,3 +288,18 @@ def test_attention_fp16_gpu_odd_batch_pitch(dev):
     ref = cuda.GpuTensor(t.clone(memory_format=torch.contiguous_format).reshape(1, H, S, D))
     got = cuda.attention_fp16_gpu(g, g, g).tensor
     assert torch.equal(got, cuda.attention_fp16_gpu(ref, ref, ref).tensor)
+
+
+@pytest.mark.parametrize("B,H,S,Sk", [(1, 3, 16, 256), (1, 3, 16, 257), (32, 3, 7, 384),
+                                      (2, 3, 100, 700), (26, 5, 65, 700)])
+def test_attention_fp16_gpu_long_keys(dev, B, H, S, Sk):
+    """K and V longer than Q, on both sides of the one-launch rule, against the
+    fp16 attention of the converted tensors."""
+    from zenith_amd import core_cuda as cuda
+    from zenith_amd import zenith_cuda as zc
+
+    q, k, v = (torch.from_numpy(synthetic.normal((B, H, n, 64), tag=80 + i)).to(dev)
+               for i, n in enumerate((S, Sk, Sk)))
+    got = cuda.attention_fp16_gpu(*(cuda.GpuTensor(t) for t in (q, k, v))).tensor
+    ref = zc.flash_attention(q.half(), k.half(), v.half()).float()
+    torch.testing.assert_close(got, ref, rtol=2.0**-10, atol=2.0**-24)

@@ -205,14 +205,22 @@ def _attn_fp16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> GpuTensor:
     """fp16 attention on fp32 tensors: one launch for up to 128 queries of
     dim 64, else converted, computed and converted back."""
     B, H, S, D = q.shape
-    # contiguous by GpuTensor; a dimension of one may carry any stride all the same
-    if D == 64 and S <= 128 and all(t.data_ptr() % 16 == 0 and
-                                    all(d % 4 == 0 for d in t.stride()[:3]) for t in (q, k, v)):
+    Sk = k.shape[2]
+    # Every query block loads and rounds all of K and V again: that pays up to 256
+    # keys (384 from 96 heads), or where there are 256 workgroups of 64 queries
+    # (with fewer the launch takes blocks of 16). Converted / one launch, us, h12:
+    # b1 s128 on 128 keys 12.1 / 8.3, 256 14.2 / 13.4, 384 17.4 / 19.0, 4096 85 / 313;
+    # b8 s40 on 384 22.9 / 19.6, 512 26 / 42; b32 s128 on 4096 309 / 210.
+    # GpuTensors are contiguous, but a dimension of one may carry any stride.
+    if (D == 64 and S <= 128
+            and (Sk <= (384 if B * H >= 96 else 256) or (S + 63) // 64 * H * B >= 256)
+            and all(t.data_ptr() % 16 == 0 and all(d % 4 == 0 for d in t.stride()[:3])
+                    for t in (q, k, v))):
         o = _new(q)
         strides = L.strides_arg([*q.stride()[:3], *k.stride()[:3], *v.stride()[:3],
                                  *o.stride()[:3]])
         L.call("zk_flash_attn_fwd_f16_io32", q.data_ptr(), k.data_ptr(), v.data_ptr(),
-               o.data_ptr(), B, H, S, k.shape[2], D, strides, None, 1.0 / math.sqrt(D), _stream(q))
+               o.data_ptr(), B, H, S, Sk, D, strides, None, 1.0 / math.sqrt(D), _stream(q))
         return GpuTensor(o)
     return _to32(_attn(_to16(q), _to16(k), _to16(v), L.ZK_F16))
 
