@@ -200,6 +200,32 @@ def test_flash_attention_mask_whole_tiles(dev, S, D):
         assert ok, worst
 
 
+@pytest.mark.parametrize("B,S,D", [(16, 300, 64), (20, 300, 64), (18, 260, 48), (20, 268, 40)])
+def test_flash_attention_mask_launches(dev, B, S, D):
+    """The launches of masked batches past one round of 128-query workgroups
+    (64 queries each; mask bytes read inside the tile) against the sequences
+    one by one, which take the ordinary one: equal, and within the fp16 bar of
+    the oracle. Rows end 4, 8 and 12 bytes into a 16-byte vector."""
+    from zenith_amd import zenith_cuda as zc
+
+    H = 12
+    g = torch.Generator(device=dev).manual_seed(S + D)
+    t = [torch.randn(B, H, S, D, generator=g, device=dev).half() for _ in range(3)]
+    i = torch.arange(S, device=dev)
+    mask = torch.rand(B, 1, S, S, generator=g, device=dev) > 0.5
+    mask[1] = i[:, None] >= i[None]
+    mask[2] = i[None] < 70
+    mask[3, :, 5] = False
+    o = zc.flash_attention(*t, attn_mask=mask)
+    for b in range(B):
+        one = zc.flash_attention(*(x[b:b + 1] for x in t), attn_mask=mask[b:b + 1])
+        assert torch.equal(o[b], one[0]), b
+    q, k, v = (x[:4, :1].float().cpu().numpy() for x in t)
+    ok, worst = fp16_tol(o[:4, :1].float().cpu().numpy(),
+                         ops.attention(q, k, v, None, mask=mask[:4].cpu().numpy()))
+    assert ok, worst
+
+
 def test_flash_attention_mask_rejects_float_masks(dev):
     from zenith_amd import zenith_cuda as zc
 

@@ -64,7 +64,7 @@ __device__ __forceinline__ int kv_swz16(int r) {
 // MASK: p.mask is applied on top of the valid lengths. A tile can then be
 // fully masked for a query that has seen no valid key yet (running max still
 // -inf); the rescale factor and the exponent are guarded for that case.
-template <int D, int NW, bool PAD = false, bool MASK = false>
+template <int D, int NW, bool PAD = false, bool MASK = false, bool LEAN = false>
 __global__ __launch_bounds__(NW * 64) void fa_fwd_f16_kernel(AttnParams p) {
   constexpr int KT = 64;
   constexpr int NT = NW * 64;
@@ -131,11 +131,14 @@ __global__ __launch_bounds__(NW * 64) void fa_fwd_f16_kernel(AttnParams p) {
   // tile ahead. A wavefront whose queries keep no key of the tile skips it,
   // and one whose queries keep all of them does not apply the mask (the
   // tiles of a padding or causal mask but the few on its edge). b8 h12 s384
-  // 23.7 -> 18.3 us, b16 h12 s512 59 -> 39, b4 h12 s1024 57 -> 38.5. At D = 128
+  // 23.7 -> 17.1 us, b16 h12 s512 57 -> 35, b4 h12 s1024 54 -> 36. At D = 128
   // the registers for it cost more than it gives (b8 h12 s512 35 -> 46): the
-  // bytes are read where they are used.
-  constexpr bool AHEAD = MASK && D <= 64;
-  uint32_t raw[8], mw[8];
+  // bytes are read where they are used, as in LEAN (see the launch).
+  // A masked key's V counts with probability 0 where its tile is walked and not
+  // at all where it is skipped: rows of V that hold an infinity or NaN must not
+  // be relied on to reach the output, nor not to.
+  constexpr bool AHEAD = MASK && D <= 64 && !LEAN;
+  uint32_t raw[8], mw[2];
   if (ntiles > 0) {
     load_kv(0);
     if constexpr (AHEAD) mask_load32(p, mrow, 0, lane, raw);
@@ -145,15 +148,12 @@ __global__ __launch_bounds__(NW * 64) void fa_fwd_f16_kernel(AttnParams p) {
     stash_kv();
     bool any = true, apply = false;
     if constexpr (AHEAD) {
-      mask_words32(p, raw, mw);
-      uint32_t kept = 0, zero = 0;
-#pragma unroll
-      for (int w = 0; w < 8; ++w) {
-        kept |= mw[w];
-        zero |= (mw[w] - 0x01010101u) & ~mw[w] & 0x80808080u;  // nonzero: a byte is 0
-      }
-      any = __builtin_amdgcn_ballot_w64(kept != 0) != 0;
-      apply = __builtin_amdgcn_ballot_w64(zero != 0) != 0;
+      const uint32_t bits = mask_bits32(raw);
+      any = __builtin_amdgcn_ballot_w64(bits != 0) != 0;
+      apply = __builtin_amdgcn_ballot_w64(bits != 0xffffffffu) != 0;
+      const auto both = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+      mw[0] = both[0] >> h32;  // keys 0 .. 31 of the tile, 4 h32 on
+      mw[1] = both[1] >> h32;  // keys 32 .. 63
     }
     __syncthreads();
     if (t + 1 < ntiles) {
@@ -163,7 +163,10 @@ __global__ __launch_bounds__(NW * 64) void fa_fwd_f16_kernel(AttnParams p) {
     if constexpr (AHEAD) {
       if (any)
         attn32_tile<D, SWZ, KLD, true>(Ks, Vs, qf, t, L, p.scale_log2,
-                                       [&](int w) { return mw[w]; }, apply, lane, o, m, l);
+                                       [&](int w) {
+                                         return (mw[w >> 2] >> (2 * (w & 3))) & 0x01010101u;
+                                       },
+                                       apply, lane, o, m, l);
     } else if constexpr (MASK) {
       attn32_tile<D, SWZ, KLD, true>(
           Ks, Vs, qf, t, L, p.scale_log2,
@@ -841,6 +844,27 @@ static void launch_f16_m(const AttnParams &p, hipStream_t s) {
       return;
     }
   }
+  // Masks at D = 64: a CU holds two workgroups of 128 queries (200 registers),
+  // four of 64, or three of 128 that read their mask bytes inside the tile
+  // (LEAN, 162). Past one round of the first the others where they still fit in
+  // one. us, random / causal / lengths mask, h12: b16 s300, 576 workgroups of 128
+  // or 960 of 64: 26.8 / 22.8 / 23.3 -> 19.6 / 17.7 / 18.2; b24 s192 19.1 / 17.0 /
+  // 17.7 -> 13.8 / 12.2 / 13.0; LEAN: b20 s300 27.6 / 25.6 / 26.1 -> 22.5, b12 s500
+  // 40.1 / 36.3 / 34.0 -> 32.5. Rows of whole 64-byte lines gain less from it
+  // than from skipping tiles (b16 s384 32.6 / 26.4 / 28.7, LEAN 30.5).
+  if constexpr (MASK && D == 64) {
+    const int64_t bh = (int64_t)p.H * p.B, w4 = (p.Sq + 127) / 128 * bh, w2 = (p.Sq + 63) / 64 * bh;
+    if (w4 > 512 && w2 <= 1024) {
+      dim3 grid((unsigned)((p.Sq + 63) / 64), (unsigned)p.H, (unsigned)p.B);
+      fa_fwd_f16_kernel<D, 2, PAD, MASK><<<grid, 128, 0, s>>>(p);
+      return;
+    }
+    if (p.Sq >= 128 && w4 > 512 && w4 <= 768 && p.Sk % 64 != 0) {
+      dim3 grid((unsigned)((p.Sq + 127) / 128), (unsigned)p.H, (unsigned)p.B);
+      fa_fwd_f16_kernel<D, 4, PAD, MASK, true><<<grid, 256, 0, s>>>(p);
+      return;
+    }
+  }
   if (p.Sq >= 128) {
     dim3 grid((unsigned)((p.Sq + 127) / 128), (unsigned)p.H, (unsigned)p.B);
     fa_fwd_f16_kernel<D, 4, PAD, MASK><<<grid, 256, 0, s>>>(p);
@@ -929,8 +953,6 @@ static int attn_impl(const char *who, const void *Q, const void *K, const void *
     if (reinterpret_cast<uintptr_t>(mask) & 3u)
       return fail(ZK_ERR_UNSUPPORTED, "%s: mask must be 4-byte aligned", who);
   }
-  p.mask16 = mask && seq_k % 16 == 0 && aligned16(mask) && p.sm[0] % 16 == 0 &&
-             p.sm[1] % 16 == 0 && p.sm[2] % 16 == 0;
   p.scale_log2 = scale * 1.4426950408889634f;
   hipStream_t s = as_stream(stream);
   if (f32_io) {

@@ -19,7 +19,6 @@ struct AttnParams {
   // contiguous, every row 4-byte aligned (read 4 keys at a time).
   const uint8_t *mask;
   int64_t sm[3];
-  int mask16;  // mask rows start on 16 bytes and hold whole 16-byte vectors
   float scale_log2;  // softmax scale * log2(e)
 };
 
@@ -32,42 +31,41 @@ __device__ __forceinline__ uint32_t mask4(const AttnParams &p, const uint8_t *ro
   return k0 < p.Sk ? *(const uint32_t *)(row + k0) : 0u;
 }
 
-// The mask bytes of the 32-query wavefront's lane for tile t, in two steps so
-// that the loads of one tile can be in flight under another's work: the raw
-// words, and the lane's words as attn32_softmax_max takes them. With mask16
-// lane l loads 32 bytes of its row, keys 32 (l / 32) .. +31, and one
-// v_permlane32_swap per pair of words deals them out.
+// The mask of the 32-query wavefront's lane for tile t, in two steps so that the
+// loads of one tile can be in flight under another's work: the bytes as loaded,
+// and one bit for each. Lane l loads 32 bytes of its row, keys 32 (l / 32) .. +31
+// (a v_permlane32_swap then gives both halves of the wavefront both words).
+// The loads are 16 bytes wide from rows on any 4-byte boundary (a global load
+// needs no more), word by word only where they would pass the row's end: eight
+// single words in every tile cost rows of no whole 16-byte vectors up to a
+// third of the kernel (b8 h12 s500 28 -> 25 us, b4 h12 s1000 48 -> 43).
 __device__ __forceinline__ void mask_load32(const AttnParams &p, const uint8_t *row, int t,
                                             int lane, uint32_t (&raw)[8]) {
-  const int h32 = lane >> 5;
-  if (p.mask16) {
-    const int k0 = t * 64 + 32 * h32;
+  typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  const int k0 = t * 64 + 32 * (lane >> 5);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      u32x4 v = {0u, 0u, 0u, 0u};
-      if (k0 + 16 * h < p.Sk) v = *(const u32x4 *)(row + k0 + 16 * h);
+  for (int h = 0; h < 2; ++h) {
+    const int k = k0 + 16 * h;
+    u32x4u v = {0u, 0u, 0u, 0u};
+    if (k + 16 <= p.Sk) {
+      v = *(const u32x4u *)(row + k);
+    } else if (k < p.Sk) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) raw[4 * h + j] = v[j];
+      for (int j = 0; j < 4; ++j) v[j] = mask4(p, row, k + 4 * j);
     }
-  } else {
 #pragma unroll
-    for (int w = 0; w < 8; ++w)
-      raw[w] = mask4(p, row, t * 64 + 32 * (w >> 2) + 8 * (w & 3) + 4 * h32);
+    for (int j = 0; j < 4; ++j) raw[4 * h + j] = v[j];
   }
 }
-__device__ __forceinline__ void mask_words32(const AttnParams &p, const uint32_t (&raw)[8],
-                                             uint32_t (&mw)[8]) {
-  if (p.mask16) {
+// The 32 loaded bytes as one bit each: byte b of word i in bit 8 b + i.
+__device__ __forceinline__ uint32_t mask_bits32(const uint32_t (&raw)[8]) {
+  uint32_t bits = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const auto r = __builtin_amdgcn_permlane32_swap(raw[2 * j], raw[2 * j + 1], false, false);
-      mw[j] = r[0];
-      mw[4 + j] = r[1];
-    }
-  } else {
-#pragma unroll
-    for (int w = 0; w < 8; ++w) mw[w] = raw[w];
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t nz = (((raw[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | raw[i]) & 0x80808080u;
+    bits |= nz >> (7 - i);
   }
+  return bits;
 }
 
 __device__ __forceinline__ int valid_len(const AttnParams &p, int b) {
