@@ -101,6 +101,7 @@ def test_linear_epilogues(dev, act, M, K, N):
     (3990, 2056, 740),  # 128x96, 4x1 waves, 3-stage ring
     (6000, 2056, 750),  # 128x96, 4x1 waves, 2-stage ring
     (4700, 200, 760),   # 128x128 at N <= 1024
+    (6150, 136, 1000),  # the same, two workgroups per CU
     (4600, 72, 3000),   # 256x256 in one round
     (2050, 136, 2300),  # 128x96, two workgroups per CU
 ])

@@ -141,8 +141,11 @@ static void launch_frag_res_stats(GemmParams p, hipStream_t s) {
 //     26.2 / 32.8, 4096 28.8 / 31.2 / 28.8 / 32.7, 4608 43.6 / 33.1 / 50.9 /
 //     35.8, 6144 45 / 52 / 51.6 / 38.0; int8 keeps the 128x96 tiles, measured
 //     in the encoder). Short K: 64x64 up to three tiles per CU, then 128x128
-//     or 128x96 (M x 768 x 768; 64x64 / 128x128 / 128x96: 4608 11.9 / 10.8 /
-//     12.1, 6144 15.4 / 14.8 / 12.7, 8192 17.9 / 15.4 / 14.1).
+//     or 128x96 in one round (M x 768 x 768; 64x64 / 128x128 / 128x96: 4608 11.9 /
+//     10.8 / 12.1, 6144 15.4 / 14.8 / 12.7, 8192 17.9 / 15.4 / 14.1; where 96 and
+//     192 do not divide N, 64x64 / 128x128 / 256x192: 12288 x 512 x 512 13.4 / 12.5 /
+//     15.3, 6144 x 1024 x 1024 22.9 / 20.3 / 24.7, 7000 x 1024 x 512 16.3 / 14.5 /
+//     18.5).
 static int pick_cfg(int M, int N, int K, bool f16) {
   if (forced_cfg() >= 0) return forced_cfg();
   auto tiles = [&](int bm, int bn) {
@@ -165,7 +168,7 @@ static int pick_cfg(int M, int N, int K, bool f16) {
     return t96 <= 512 ? 6 : 5;
   }
   if (!f16 || tiles(64, 64) <= 768) return 3;
-  return t128 <= 256 ? 1 : t96 <= 512 ? 6 : 5;
+  return t128 <= 256 ? 1 : t96 <= 512 ? 6 : t128 <= 512 ? 1 : 5;
 }
 
 // Every 32x32-MFMA tile has the fragment-ordered store; the 16x16 ones give
@@ -177,8 +180,10 @@ static int frag_cfg(int cfg) { return cfg == 2 ? 1 : cfg == 3 || cfg == 7 ? 4 : 
 // HBM: four stages, all requested at the start. BERT encoder, s128, 12 layers,
 // ring of 2 / 3 / 4 / 6 stages: b1 502 / 463 / 461 / 470 us, b2 554 / 471 /
 // 459 / 473, b4 604 / 525 / 527 / 654 (6 stages leave one workgroup per CU).
-// More workgroups hide each other's: 4096x768x768 (768 tiles) 10.0 / 10.8 /
-// 12.0 us. The sums and their order are the same.
+// (b8 s128 with it for the split products alone 818, for all 796.) More
+// workgroups hide each other's: 4096x768x768 (768 tiles) 10.0 / 10.8 / 12.0 us.
+// Called over and over on the same weights it costs 0.2 to 0.4 us (2048x768x768,
+// ring of 2 / 4: 7.4 / 7.7). The sums and their order are the same.
 template <class OP, typename OutT, bool DEQ>
 [[nodiscard]] static bool launch_64(GemmParams p, int epi, hipStream_t s) {
   const int64_t wgs = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * (p.splits > 1 ? p.splits : 1);
