@@ -189,7 +189,7 @@ def test_matmul_broadcast_operands(dev, M, K, N):
 
 
 @pytest.mark.parametrize("M,K,N", [
-    (4100, 72, 4100),   # bf16 split, 128x64 tile
+    (4100, 72, 4100),   # bf16 split, 64x64 tile
     (4000, 100, 2000),
     (520, 200, 20500),
     (700, 136, 1100),   # 198 tiles: 64x64 fp32 MFMA
@@ -304,8 +304,11 @@ def test_matmul_fp32_wide_b(dev, M, K):
     (64, 1100, 1600, 0),   # 64x64 tile, K split, K a multiple of 32
     (65, 127, 1001, 3),    # rows off 16 bytes, one row and one k past a tile
     (1500, 1030, 36, 0),   # 64x64 unsplit, the K tail one vector
-    (2050, 2017, 100, 4),  # 128x64 tile, ragged in M and N
-    (4100, 1030, 33, 0),   # 128x64, a K tail of one value
+    (2050, 2017, 100, 4),  # 64x64 in two rounds, ragged in M and N
+    (4100, 1030, 33, 0),   # the same, a K tail of one value
+    (1930, 2017, 100, 4),  # 128x64 tile, ragged in M and N
+    (3650, 1030, 33, 0),   # 128x64, a K tail of one value
+    (5000, 2017, 36, 4),   # 128x64 for B[K,N], 64x64 for W[N,K]
 ])
 def test_gemm_f32_bf16_split(dev, trans_b, M, N, K, pad):
     """The bf16-split fp32 GEMM in both layouts, with and without a
@@ -386,15 +389,15 @@ def test_gemm_f32_bf16_split_small_values(dev, trans_b, exp_a, exp_b):
 
 
 @pytest.mark.parametrize("trans_b", [True, False])
-@pytest.mark.parametrize("N", [1100, 1030])  # rows of whole 16-byte vectors, and not
+@pytest.mark.parametrize("M,N", [(1100, 1100), (1100, 1030), (1930, 2017)])  # both tiles; rows off 16 bytes
 @pytest.mark.parametrize("K", [40, 3201])  # one slice and a tail; K split
-def test_gemm_f32_bf16_split_large_values(dev, trans_b, N, K):
+def test_gemm_f32_bf16_split_large_values(dev, trans_b, M, N, K):
     """Sums and products up to FLT_MAX: finite wherever fp32's are, and infinite
     where the result is past its range. Rows 0 to 127 hold products within 2^-9
     of FLT_MAX whose factors' leading bf16 parts multiply past it."""
     from zenith_amd import _lib as L
 
-    M, fmax = 1100, float(np.finfo(np.float32).max)
+    fmax = float(np.finfo(np.float32).max)
     rng = np.random.default_rng(K)
     a = np.ldexp(rng.uniform(1, 2, (M, K)), rng.integers(40, 58, (M, 1))).astype(np.float32)
     b = np.ldexp(rng.uniform(-2, 2, (K, N)), rng.integers(40, 58, (1, N))).astype(np.float32)
