@@ -221,6 +221,7 @@ def test_linear_fp32_tile_configs(dev, M, K, N):
     (130, 200, 1600, 0),     # 64x64, K split (with a workspace)
     (2000, 2040, 72, 8),     # 128x128 tile
     (4090, 2296, 64, 0),     # 256x192 tile, one slice
+    (100, 31000, 72, 8),     # few rows, many columns: 128x128
     (4100, 4072, 200, 8),    # 256x256 tile
 ])
 @pytest.mark.parametrize("out", [torch.float32, torch.float16])

@@ -26,15 +26,18 @@ void launch_nn(GemmParams p, hipStream_t s) {
 // 64x64): 4096^3 129 / 171 / 146 / 212; 4096x2304x768 30.6 / 27.3 / 28.5 /
 // 29.8; 3000x2000x1504 43 / 38 / 31 / 43; 2048^3 50 / 44 / 30.7 / 30.6;
 // 4096x768x768 24 / 21 / 13.6 / 12.6. The transpose that went before each of
-// them took 5 to 20 us.
+// them took 5 to 20 us. Up to 128 rows a 256-row tile is at least half empty
+// (256x192 / 128x128 or 64x64: 64x32000x768 21.8 / 14.4, 16x50264x768 36.2 / 21.4,
+// 128x128000x4096 263 / 250; from 129 it is level or ahead: 129x32000x768 23.6 /
+// 27.0).
 template <typename OutT>
 void run_nn(GemmParams p, hipStream_t s) {
   const int64_t tm = (p.M + 255) / 256, t256 = tm * ((p.N + 255) / 256),
                 t192 = tm * ((p.N + 191) / 192),
                 t128 = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
-  if (t256 >= 256 && (t192 + 255) / 256 * 3 >= (t256 + 255) / 256 * 4)
+  if (p.M > 128 && t256 >= 256 && (t192 + 255) / 256 * 3 >= (t256 + 255) / 256 * 4)
     launch_nn<256, 256, 32, 2, 4, OutT>(p, s);
-  else if (t192 >= 160)
+  else if (p.M > 128 && t192 >= 160)
     launch_nn<256, 192, 32, 4, 2, OutT>(p, s);
   else if (t128 >= 256)
     launch_nn<128, 128, 32, 2, 2, OutT>(p, s);
