@@ -171,9 +171,11 @@ int zk_gemm_f16_nn(const void *A, const void *B, void *C, int64_t M, int64_t N, 
 
 /* FP32 GEMM, C[M,N] = A[M,K] . op(B), trans_b as above, at fp32 precision
  * with fp32 accumulation: fp32 MFMA products, or each operand split exactly
- * into three bf16 parts whose products of weight 2^-16 and above run on the
- * bf16 MFMA (an error against 64 bits no larger than the fp32 products'),
- * or the SIMT kernel for the smallest.
+ * (subnormals included) into three bf16 parts whose products of weight 2^-16
+ * and above run on the bf16 MFMA (an error against 64 bits no larger than the
+ * fp32 products'), or the SIMT kernel for the smallest. Infinities, NaN and
+ * sums up to FLT_MAX as in fp32 products; where a 64-row block has a sum past
+ * 2^96, or a value that is not finite, it is formed a second time on fp32 MFMA.
  * Replaces zenith_cuda.matmul (cuda_bindings.cpp:73-88 ->
  * matmul_f32 cuda_kernels.cu:297-336, 524-528). */
 int zk_gemm_f32(const float *A, const float *B, float *C, int64_t M,

@@ -36,10 +36,11 @@
 // start on 16 bytes; otherwise the Python layer transposes it once
 // (zk_transpose_f16).
 //
-// zk_gemm_f32: small W[N,K] products run the same kernel on fp32 matrix
-// instructions, larger ones and B[K,N] the bf16-split kernel of
-// zk_gemm_f32s.hip, the rest an fp32 SIMT kernel (64x64 tiles, 4x4 outputs per thread) for
-// the reference's fp32 `matmul` entry point, which must stay exact fp32.
+// zk_gemm_f32 (the reference's fp32 `matmul`): small W[N,K] products run the
+// same kernel on fp32 matrix instructions, larger ones and B[K,N] the
+// bf16-split kernel of zk_gemm_f32s.hip, whose error against 64 bits is no
+// larger than theirs, the rest an fp32 SIMT kernel (64x64 tiles, 4x4 outputs
+// per thread).
 #include <type_traits>
 
 #include "zk_gemm_kernel.hpp"

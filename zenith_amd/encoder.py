@@ -353,7 +353,10 @@ class BertEncoder:
                    scale, stream)
         else:
             # QKV whole: its split's reduction launch costs more than the split saves
-            # (b1 s128 460 -> 432 us per step; from b2 on it does not split)
+            # wherever it would split, below 128 tiles of 64 x 64 (12 layers, us, split /
+            # whole: hidden 768, 16 rows 371 / 359, 64 435 / 412, 128 455 / 427, 192 483 /
+            # 454; hidden 256, 512 rows 450 / 410; 512, 128 rows 453 / 412; 1024, 64 rows
+            # 488 / 484, 128 516 / 501)
             self._gemm(x, w["Wqkv"], w["bqkv"], qkv, L.ZK_EPI_BIAS, stream=stream, split=False)
             self._attention(qkv, ctx, lens, B, S, stream)
         if self.int8 is None:

@@ -438,9 +438,11 @@ def flash_attention(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor,
     j >= length; `attn_mask` (bool, broadcastable to [batch, heads, seq_q,
     seq_k], True = attend: scaled_dot_product_attention's boolean mask) masks
     any (query, key) pair; both may be given. Masked keys get probability
-    exactly 0 and a query with no key left returns 0. fp32 and fp16; any
-    head_dim up to 128 (HEAD_DIM_MAX, flash_attention.cu:26); fp16 head_dims
-    that are not a multiple of 8 are zero-padded to one."""
+    exactly 0 and a query with no key left returns 0; their rows of V must be
+    finite all the same (0 times an infinity or NaN may or may not reach the
+    output). fp32 and fp16; any head_dim up to 128 (HEAD_DIM_MAX,
+    flash_attention.cu:26); fp16 head_dims that are not a multiple of 8 are
+    zero-padded to one."""
     if not Q.is_cuda:
         raise RuntimeError("Q must be CUDA tensor")
     _need_cuda(Q, K, V, key_padding_lengths, attn_mask)
