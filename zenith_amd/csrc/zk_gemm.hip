@@ -131,7 +131,9 @@ static void launch_frag_res_stats(GemmParams p, hipStream_t s) {
 //     256x256 that fits in one of one per CU (M x 3072 x 768, erf-GELU;
 //     128x96 / 128x128 / 256x192 / 256x256: M 1577 15.8 / 17.6 / 22.1 / 26.1,
 //     2560 24.3 / 19.7 / 23.0 / 26.9, 3500 28.9 / 28.2 / 24.5 / 28.2, 4608
-//     37.4 / 34.1 / 43.6 / 30.1);
+//     37.4 / 34.1 / 43.6 / 30.1; int8, re-quantising, the same order: 16.6 / 17.2 /
+//     23.4 / 28.8, 25.2 / 18.5 / 24.6 / 29.8, 30.1 / 27.2 / 25.8 / 30.9, 37.6 / 32.5 /
+//     46.3 / 31.6);
 //   from 256 tiles of 256x256: that tile, unless 256x192 takes fewer whole
 //     rounds times area (QKV at s512, 16384 x 2304: 576 tiles of 256x256, three
 //     rounds with the last a quarter full, or 768 of 256x192);
