@@ -681,7 +681,9 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_f32_kernel(AttnParams p) {
     // subnormals: such a key still counts where its V is large. What the
     // instruction left out of this stage is formed again and added here, after
     // it and one key block at a time, which costs stages that need none 0.4% on
-    // average (D = 64: 2%; b4 h12 s256 14.9 -> 15.3 us). exp2f throughout costs 3
+    // average (D = 64: 2%; b4 h12 s256 14.9 -> 15.3 us). Scores so far apart that
+    // every stage takes it (q 15 times N(0, 1)): b4 h12 s256 26.5 us, b4 h16 s1024
+    // d128 560 (299 otherwise; 1340 on the FMA pipe). exp2f throughout costs 3
     // to 9%, a branch before the products 5 to 7% of the short chains, a second
     // pass over all keys at the end 1.6%; with the scores held or the blocks
     // unrolled here D = 128 spills.
